@@ -259,10 +259,10 @@ int vbsr_launch_split_row(const vbsr_matrix* matrix, const float* B, float* C, i
 int vbsr_launch_split_row_static(const vbsr_matrix* matrix, const float* B, float* C, int32_t rhs,
                                  hipStream_t stream);
 
-/* launch_row_owned_scalar (vbsr.hpp:161; row_owned.cu:376-395): one output
- * per lane, accumulated with fmaf over blocks in row_ptr order and k
- * ascending from 0 -- the reference kernels' exact order, so its results are
- * bit-identical to theirs. */
+/* launch_row_owned_scalar (vbsr.hpp:161; row_owned.cu:376-395): every output
+ * is one fmaf chain over blocks in row_ptr order and k ascending from 0 --
+ * the reference kernels' exact order, so its results are bit-identical to
+ * theirs. */
 int vbsr_launch_row_owned_scalar(const vbsr_device_view* matrix, const float* B, float* C,
                                  int32_t rhs, hipStream_t stream);
 

@@ -1,0 +1,67 @@
+"""GPU kernels at the sizes where their tilings and dispatch rules change, against the CPU oracle.
+
+Shares test_gpu_parity's bounds: the order-preserving kernel bit for bit against the oracle's fmaf emulation, the
+MFMA kernels within the elementwise FP32 bound and bit-identical across runs.
+"""
+
+import numpy as np
+import pytest
+
+import oracle_ffi as o
+import test_gpu_parity as parity
+import varblockspmm_amd as vb
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+
+def bits(a):
+    return np.asarray(a, dtype=np.float32).view(np.uint32)
+
+
+# Blocks per row on both sides of the order-preserving kernel's metadata segments (64 blocks), then row counts on
+# both sides of its XCD runs (rows / 64 consecutive rows, at most 64), with heights and widths cycling through 8..64.
+ORDERED_ROWS = {f"blocks-{n}": [n, 0, 1] for n in (1, 63, 64, 65, 129)}
+ORDERED_ROWS.update({f"rows-{n}": [i % 4 for i in range(n)] for n in (1, 7, 9, 63, 65, 127, 129, 1031, 4161)})
+
+
+@pytest.mark.parametrize("rhs", [8, 16, 32, 64])
+@pytest.mark.parametrize("name", list(ORDERED_ROWS))
+def test_ordered_kernel_at_segment_and_run_edges(name, rhs):
+    degrees = ORDERED_ROWS[name]
+    parity.note(f"ordered {name} rhs={rhs}")
+    host = parity.hand_made([8 * (1 + (3 * i + 7) % 8) for i in range(len(degrees))],
+                            [8 * (1 + (5 * j + 2) % 8) for j in range(131)],
+                            [[(7 * i + j) % 131 for j in range(d)] for i, d in enumerate(degrees)])
+    c = parity.Case(host, rhs, 23)
+    np.testing.assert_array_equal(bits(c.run_scalar()), bits(o.fmaf_order(c.oracle, c.b, rhs)))
+    c.close()
+
+
+def extreme_case(a_exponent, b_exponent, rhs):
+    """A small matrix whose values (and B) are uniform in [-1, 1] times powers of two."""
+    host = parity.hand_made([8, 24, 64], [40, 8, 16], [[0, 1], [2], [1, 0, 2]], seed=4)
+    host.values = np.ldexp(host.values, a_exponent).astype(np.float32)
+    b = np.ldexp(o.make_random_input(host.scalar_cols * rhs, 29), b_exponent).astype(np.float32)
+    return host, b
+
+
+@pytest.mark.parametrize("rhs", [8, 32])
+@pytest.mark.parametrize("a_exponent, b_exponent, found", [
+    (-140, 0, "subnormal"),   # subnormal values
+    (-67, -67, "subnormal"),  # every product below 2^-134, the least normal number being 2^-126
+    (64, 64, "infinite"),     # products up to 2^128, past the largest finite number
+])
+def test_ordered_kernel_keeps_the_bits_of_extreme_values(a_exponent, b_exponent, found, rhs):
+    parity.note(f"extreme 2^{a_exponent} * 2^{b_exponent} rhs={rhs}")
+    host, b = extreme_case(a_exponent, b_exponent, rhs)
+    c = parity.Case(host, rhs, 29)
+    want = o.fmaf_order(c.oracle, b, rhs)
+    assert np.any(np.isinf(want)) if found == "infinite" else np.any((want != 0) & (np.abs(want) < 2.0 ** -126))
+    c.b_dev = torch.from_numpy(b).to(parity.DEVICE)
+    got = c.run_scalar()
+    nan = np.isnan(want)  # inf - inf: which NaN is not defined
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(bits(got)[~nan], bits(want)[~nan])
+    c.close()

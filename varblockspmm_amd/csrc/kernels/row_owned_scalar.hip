@@ -4,16 +4,38 @@
 // Every output C[r, n] is one fmaf chain: acc = 0, then for each block of the
 // row in row_ptr order and k ascending, acc = fmaf(A[r, k], B[k, n], acc).
 // That is the order every reference kernel uses, so this kernel's results
-// are bit-identical to the reference's.  It is the GPU-side order oracle and
-// the profiling baseline, not the fast path.
+// are bit-identical to the reference's.  It is the GPU-side order oracle.
 //
-// Mapping: one workgroup per block row.  Lane (r, g) owns local row r and
-// the adjacent output columns of group g: 4 groups of RHS/4 columns (256
-// lanes), or 8 groups of 8 at RHS 64 (512 lanes), so gh lanes cover the row
-// in one pass and each A value a lane loads feeds RHS/groups fmaf chains.
-// Each block's B slice (w x RHS floats) is staged once per workgroup in LDS,
-// double-buffered with one barrier per block, stored k-major with a padded
-// row (RHS + 4 floats) so a lane's columns are one 8- to 64-byte read.
+// Arithmetic.  v_mfma_f32_16x16x4_f32 accumulates exactly like four fmafs,
+// k = 0, 1, 2, 3 in turn, each rounded (measured against fmaf, bit for bit:
+// 1M outputs each of ordinary values, 30 binades of exponents, subnormal
+// results, overflow, signed zeros and arbitrary bit patterns with NaNs; the
+// reversed order differs), so a chain of MFMAs over ascending k is the fmaf
+// chain.  Tiles are transposed, D[n][r] = sum_k B[k, n] * A[r, k]: MFMA i of a
+// step at k0 takes k0 + 4 i .. k0 + 4 i + 3, lane 16 g + x supplying
+// B[k0 + 4 i + g, n0 + x] and A[r0 + x, k0 + 4 i + g], and result register v
+// of that lane is C[r0 + x, n0 + 4 g + v].  A step is 16 columns of a block;
+// the 8 columns that end a block whose width is 8 mod 16 take two MFMAs
+// instead of four, so no zero is ever added to a chain.
+//
+// Mapping.  One workgroup of 4 waves per block row.  An output's chain cannot
+// be split, so the waves share the row's 16 x 16 output tiles instead: at
+// RHS 64 wave w takes RHS tile w of every row tile, at RHS 32 RHS tile w & 1
+// of every other row tile, at RHS 16 and 8 row tile w.  A step's A columns
+// (contiguous, 64 h bytes) and its B slice are loaded once per workgroup, 16
+// and RHS / 4 bytes per thread, kStages - 1 steps ahead in registers, and go
+// through two LDS buffers with one barrier per step.  Block metadata is read
+// 64 blocks at a time, one per lane.
+//
+// What bounds it.  At full size the L2-miss reads, as for the MFMA plan
+// kernel, whose time it comes within 7-22% of; for few, long rows one row's
+// chain of steps (0.36 us a step on an otherwise idle CU).  Measured at 4096
+// block rows of degree 8 (high sizes, random columns), against one fmaf per
+// output, k and lane with B broadcast from LDS, which the LDS read rate bound:
+// RHS 8 / 16 / 32 / 64 83.5 -> 42.8, 99.9 -> 47.6, 186 -> 65.1, 297 -> 106 us
+// per call.  Two stages: 300 rows of degree 16 +11%, the rest within 1%; four
+// stages: +1-3%.  Reading the next step's operands back from LDS during the
+// current step's MFMAs: -0.5% to +4%.
 #include <hip/hip_runtime.h>
 
 #include "../internal.hpp"
@@ -21,87 +43,233 @@
 namespace vbsr_amd {
 namespace {
 
-constexpr int kMaxBlockDim = 64;  // largest block height and width
+using f32x4 = float __attribute__((ext_vector_type(4)));
+using rsrc_t = __amdgpu_buffer_rsrc_t;
 
-// Column groups per local row, and the workgroup that covers 64 rows of them.
+constexpr int kWave = 64;
+constexpr int kWaves = 4;
+constexpr int kThreads = kWave * kWaves;
+constexpr int kStages = 3;     // register stages of a step's loads
+constexpr int kMaxTiles = 4;   // h <= 64
+constexpr int kRawBufferFlags = 0x00020000;
+constexpr int kNonTemporal = 2;
+
 template <int RHS>
-constexpr int scalar_groups() {
-  return RHS >= 32 ? 8 : 4;
+struct Shape {
+  static constexpr int kRhsTiles = RHS < 16 ? 1 : RHS / 16;
+  static constexpr int kWavesPerTileColumn = kWaves / kRhsTiles;  // waves that share an RHS tile's row tiles
+  static constexpr int kBVec = RHS < 16 ? 1 : RHS / 16;           // floats of B per thread and step
+  static constexpr int kBFloats = 16 * 16 * kRhsTiles;
+};
+
+// Leading dimension of the A buffer, float (r, k) at k * ld + r: 16 mod 64 or
+// 48 mod 64, so that the four lane groups, which read four consecutive k, hit
+// four disjoint quarters of the banks.
+template <int T>
+constexpr int a_ld() {
+  return T == 1 ? 16 : T == 4 ? 80 : 48;
 }
-template <int RHS>
-constexpr int scalar_threads() {
-  return scalar_groups<RHS>() * kMaxBlockDim;
+constexpr int kAFloats = 16 * a_ld<kMaxTiles>();
+
+// Float (k, n) of the B buffer: column-major, the four 16-byte pieces of a
+// column permuted by an XOR of n's bits 1-2, which keeps the writes (16 k of
+// consecutive columns) and the reads (4 k of 16 columns) free of conflicts.
+__device__ __forceinline__ int b_index(int k, int n) {
+  return n * 16 + ((((k >> 2) ^ (n >> 1) ^ (n >> 2)) & 3) << 2) + (k & 3);
 }
 
-template <int RHS>
-__global__ __launch_bounds__(scalar_threads<RHS>()) void row_owned_scalar_kernel(vbsr_device_view a,
-                                                                          const float* __restrict__ b,
-                                                                          float* __restrict__ c) {
-  constexpr int kGroups = scalar_groups<RHS>();
-  constexpr int kThreads = scalar_threads<RHS>();
-  constexpr int kCols = RHS / kGroups;  // output columns per lane
-  constexpr int kLd = RHS + 4;          // LDS row of one k of a B slice
-  __shared__ __attribute__((aligned(16))) float slice[2][kMaxBlockDim * kLd];
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-  const int row = blockIdx.x;
-  const int tid = int(threadIdx.x);
-  const int h = a.row_size[row];
+__device__ __forceinline__ int64_t lane_value(int64_t v, int lane) {
+  const int lo = __builtin_amdgcn_readlane(int(uint32_t(uint64_t(v))), lane);
+  const int hi = __builtin_amdgcn_readlane(int(uint32_t(uint64_t(v) >> 32)), lane);
+  return int64_t((uint64_t(uint32_t(hi)) << 32) | uint32_t(lo));
+}
+
+// N floats at float alignment (B panels need only be 4-byte aligned).
+template <int N>
+struct BVec {
+  typedef float type __attribute__((ext_vector_type(N)));
+  typedef float unaligned __attribute__((ext_vector_type(N), aligned(4)));
+};
+template <>
+struct BVec<1> {
+  typedef float type, unaligned;
+};
+
+template <int RHS, int T>
+__device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const float* b, float* c, int row, int h,
+                                            float* lds, int wave, int lane) {
+  using S = Shape<RHS>;
+  using bvec = typename BVec<S::kBVec>::type;
+  constexpr int ld = a_ld<T>();
+  // Row tiles of one wave: first, first + kStride, ...
+  constexpr int kStride = S::kWavesPerTileColumn;
+  constexpr int kOwn = (T + kStride - 1) / kStride;
+  const int rhs_tile = wave % S::kRhsTiles;
+  const int first_tile = wave / S::kRhsTiles;
+  const int group = lane >> 4;
+  const int x = lane & 15;
+  const int tid = wave * kWave + lane;
+
+  // A: this thread's 16 bytes of the step's column-major h x 16 tile.  f / h
+  // is (f * ceil(2^16 / h)) >> 16, exact for f < 1024 and h a multiple of 8.
+  const uint32_t h_recip = (65536u + uint32_t(h) - 1u) / uint32_t(h);
+  const int f = 4 * tid;
+  const int fk = int((uint32_t(f) * h_recip) >> 16);
+  const int a_write = fk * ld + (f - fk * h);
+  const bool a_owner = f < 16 * h;
+
+  // B: this thread's floats k .. k + kBVec - 1 of column n of the step.  A
+  // half step has no k >= 8: those threads read their column's lower half
+  // again, which no MFMA of the half step takes.
+  constexpr int kPerColumn = 16 / S::kBVec;
+  const int b_n = tid / kPerColumn;
+  const int b_k = (tid % kPerColumn) * S::kBVec;
+  const int b_col = RHS < 16 ? b_n & (RHS - 1) : b_n;
+  const float* b_lane = b + int64_t(b_col) * a.scalar_cols + b_k;
+  const int b_back = b_k >= 8 ? 8 : 0;
+  const int b_write = b_index(b_k, b_n);
+  float* a_bufs = lds;
+  float* b_bufs = lds + 2 * kAFloats;
+  int b_read[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) b_read[i] = b_index(4 * i + group, 16 * rhs_tile + x);
+  const int a_read = group * ld + 16 * first_tile + x;
+
+  f32x4 acc[kOwn];
+#pragma unroll
+  for (int j = 0; j < kOwn; ++j) acc[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
   const int first = a.row_ptr[row];
   const int last = a.row_ptr[row + 1];
-  const int r = tid % h;
-  const int g = tid / h;
-  const bool owner = g < kGroups;  // kGroups * h lanes own outputs; the rest only stage B
-
-  // Stages block blk's B slice: B[col0 + k, n] for k < w, n < RHS at k * kLd + n.
-  auto stage = [&](int blk, float* dst) {
+  int parity = 0;
+  for (int seg = first; seg < last; seg += kWave) {
+    const int blocks = min(kWave, last - seg);
+    // Lane j holds block seg + j.
+    const int blk = seg + min(lane, blocks - 1);
     const int col = a.block_col[blk];
+    const int64_t a_off = a.value_off[blk];
+    const int64_t b_off = a.col_scalar_off[col];
     const int w = a.col_size[col];
-    const float* src = b + a.col_scalar_off[col];
-    const int k = tid % kMaxBlockDim;
-    if (k < w)
-      for (int n = tid / kMaxBlockDim; n < RHS; n += kThreads / kMaxBlockDim)
-        dst[k * kLd + n] = src[k + int64_t(n) * a.scalar_cols];
-  };
 
-  float acc[kCols];
+    // The next step to load: columns k0 .. of block `at` of the segment.
+    int at = 0, k0 = 0;
+    int64_t at_a = lane_value(a_off, 0), at_b = lane_value(b_off, 0);
+    int at_w = __builtin_amdgcn_readlane(w, 0);
+    struct Stage {
+      f32x4 a;
+      bvec b;
+      int mfmas;  // 4, 2 for a half step, 0 past the segment
+    };
+    // Loads the next step.  Past the segment's end the A resource is empty
+    // and B reads the last block's first columns again; neither is used.
+    auto issue = [&](Stage& st) {
+      const bool live = at < blocks;
+      const bool half = at_w - k0 == 8;
+      st.mfmas = !live ? 0 : half ? 2 : 4;
+      const rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.values + at_a + int64_t(k0) * h),
+                                                            short(0), st.mfmas * 4 * h * 4, kRawBufferFlags);
+      st.a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * tid, 0, kNonTemporal));
+      st.b = *reinterpret_cast<const typename BVec<S::kBVec>::unaligned*>(b_lane + at_b + k0 - (half ? b_back : 0));
+      k0 += 16;
+      if (k0 >= at_w) {
+        ++at;
+        k0 = 0;
+        const int l = min(at, blocks - 1);
+        at_a = lane_value(a_off, l);
+        at_b = lane_value(b_off, l);
+        at_w = __builtin_amdgcn_readlane(w, l);
+      }
+    };
+    // Publishes the step's A and B and runs the wave's tiles.  The buffers
+    // alternate: a wave writes buffer p only after the barrier of the step
+    // before, which every wave reaches after its reads of buffer p.
+    auto compute = [&](const Stage& st) {
+      float* as = a_bufs + parity * kAFloats;
+      float* bs = b_bufs + parity * S::kBFloats;
+      parity ^= 1;
+      if (a_owner) *reinterpret_cast<f32x4*>(as + a_write) = st.a;
+      *reinterpret_cast<bvec*>(bs + b_write) = st.b;
+      __syncthreads();
+      auto mfma = [&](int i) {
+        const float bv = bs[b_read[i]];
 #pragma unroll
-  for (int j = 0; j < kCols; ++j) acc[j] = 0.0f;
+        for (int j = 0; j < kOwn; ++j)
+          if (T % kStride == 0 || first_tile + j * kStride < T)
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv, as[a_read + 4 * i * ld + 16 * j * kStride], acc[j], 0, 0, 0);
+      };
+      mfma(0);
+      mfma(1);
+      if (st.mfmas > 2) {
+        mfma(2);
+        mfma(3);
+      }
+    };
+    Stage s[kStages];
+#pragma unroll
+    for (int q = 0; q < kStages - 1; ++q) issue(s[q]);
+    for (bool more = true; more;) {
+#pragma unroll
+      for (int q = 0; q < kStages; ++q) {
+        issue(s[(q + kStages - 1) % kStages]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s[q].mfmas > 0) compute(s[q]);
+      }
+      more = s[0].mfmas > 0;
+    }
+  }
 
-  if (first < last) stage(first, slice[0]);
-  __syncthreads();
-  for (int blk = first; blk < last; ++blk) {
-    const int buf = (blk - first) & 1;
-    if (blk + 1 < last) stage(blk + 1, slice[buf ^ 1]);
-    if (owner) {
-      const int w = a.col_size[a.block_col[blk]];
-      const float* a_col = a.values + a.value_off[blk] + r;
-      const float* bs = slice[buf] + g * kCols;
-      // w is a multiple of 8: eight A loads in flight, then their fmafs in
-      // k order.
-      for (int k0 = 0; k0 < w; k0 += 8) {
-        float av[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) av[i] = a_col[int64_t(k0 + i) * h];
+  for (int j = 0; j < kOwn; ++j) {
+    const int r = 16 * (first_tile + j * kStride) + x;
+    if (r < h) {
+      float* c_row = c + a.row_scalar_off[row] + r;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float* bk = bs + (k0 + i) * kLd;
-#pragma unroll
-          for (int j = 0; j < kCols; ++j) acc[j] = __builtin_fmaf(av[i], bk[j], acc[j]);
-        }
+      for (int v = 0; v < 4; ++v) {
+        const int n = 16 * rhs_tile + 4 * group + v;
+        if (n < RHS) c_row[int64_t(n) * a.scalar_rows] = acc[j][v];
       }
     }
-    __syncthreads();
   }
-  if (owner) {
-    float* c_row = c + a.row_scalar_off[row] + r;
-#pragma unroll
-    for (int j = 0; j < kCols; ++j) c_row[int64_t(g * kCols + j) * a.scalar_rows] = acc[j];
+}
+
+// Workgroup i runs on XCD i mod 8.  Rows are dealt to the XCDs in runs of
+// `chunk` consecutive rows, so that rows that share block columns (a band
+// matrix's neighbours) share an L2; a run is at most a 64th of the rows, so
+// that rows of similar length standing together still spread over all XCDs.
+__host__ __device__ __forceinline__ int row_chunk(int rows) {
+  const int chunk = rows / (8 * kXcds);
+  return chunk < 1 ? 1 : chunk > 64 ? 64 : chunk;
+}
+__host__ __device__ __forceinline__ int row_of(int group, int rows) {
+  const int chunk = row_chunk(rows);
+  const int turn = group / (kXcds * chunk);
+  return (turn * kXcds + group % kXcds) * chunk + group / kXcds % chunk;
+}
+
+template <int RHS>
+__global__ __launch_bounds__(kThreads) void row_owned_ordered_kernel(vbsr_device_view a, const float* __restrict__ b,
+                                                                     float* __restrict__ c) {
+  __shared__ __attribute__((aligned(16))) float lds[2 * (kAFloats + Shape<RHS>::kBFloats)];
+  const int row = row_of(int(blockIdx.x), a.block_rows);
+  if (row >= a.block_rows) return;
+  const int wave = uniform(int(threadIdx.x) / kWave);
+  const int lane = int(threadIdx.x) % kWave;
+  const int h = uniform(a.row_size[row]);
+  switch ((h + 15) >> 4) {
+  case 1: ordered_row<RHS, 1>(a, b, c, row, h, lds, wave, lane); break;
+  case 2: ordered_row<RHS, 2>(a, b, c, row, h, lds, wave, lane); break;
+  case 3: ordered_row<RHS, 3>(a, b, c, row, h, lds, wave, lane); break;
+  default: ordered_row<RHS, 4>(a, b, c, row, h, lds, wave, lane); break;
   }
 }
 
 template <int RHS>
 void launch(const vbsr_device_view& a, const float* b, float* c, hipStream_t stream) {
-  row_owned_scalar_kernel<RHS><<<dim3(unsigned(a.block_rows)), dim3(scalar_threads<RHS>()), 0, stream>>>(a, b, c);
+  const int64_t turn = int64_t(kXcds) * row_chunk(a.block_rows);
+  const int64_t groups = (a.block_rows + turn - 1) / turn * turn;
+  row_owned_ordered_kernel<RHS><<<dim3(unsigned(groups)), dim3(kThreads), 0, stream>>>(a, b, c);
 }
 
 }  // namespace
