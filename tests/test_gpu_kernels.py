@@ -65,3 +65,40 @@ def test_ordered_kernel_keeps_the_bits_of_extreme_values(a_exponent, b_exponent,
     np.testing.assert_array_equal(np.isnan(got), nan)
     np.testing.assert_array_equal(bits(got)[~nan], bits(want)[~nan])
     c.close()
+
+
+@pytest.mark.parametrize("name", ["empty-repeat-unsorted", "single-row", "long-row", "packed-light"])
+@pytest.mark.parametrize("rhs", [32, 64])
+def test_columns_per_workgroup_do_not_change_the_bits(rhs, name):
+    """The split-k kernel on 16 and on 32 columns at a time, with both forms of B's addressing: within tolerance of
+    the oracle, and the same bits (a column's sums depend only on how its row's steps are dealt to the waves).  A
+    number of columns that no kernel has is refused."""
+    parity.note(f"columns {name} rhs={rhs}")
+    c = parity.Case(parity.EDGE_MATRICES[name](), rhs, 31)
+    view, results = c.matrix.device_view(), []
+    for columns in (16, 32):
+        for launch in (vb.launch_row_owned, vb.launch_row_owned_wide_b):
+            schedule = c.matrix.row_schedule()
+            schedule.rhs64_tiles = 0
+            schedule.rhs32_columns = schedule.rhs64_columns = columns
+            results.append(c.run(lambda: launch(view, schedule, c.b_dev, c.c_dev, rhs, c.stream)))
+    c.check_tolerance(results[0], name)
+    for other in results[1:]:
+        np.testing.assert_array_equal(bits(other), bits(results[0]))
+    schedule.rhs32_columns = schedule.rhs64_columns = 24
+    with pytest.raises(ValueError, match="columns per workgroup"):
+        vb.launch_row_owned(view, schedule, c.b_dev, c.c_dev, rhs, c.stream)
+    c.close()
+
+
+@pytest.mark.parametrize("rows, degree, few", [(128, 16, True), (129, 16, False), (250, 4, True), (450, 8, False)])
+def test_few_rows_take_their_columns_in_parts(rows, degree, few):
+    """Both sides of the rule (at most 128 workgroups, or 384 with at most 4096 k steps), through the plan."""
+    parity.note(f"column rule {rows} rows, degree {degree}")
+    host = vb.generate(rows, rows, degree, "high", "random", 5)
+    for rhs in (32, 64):
+        c = parity.Case(host, rhs, 37)
+        schedule = c.matrix.row_schedule()
+        assert (schedule.rhs32_columns, schedule.rhs64_columns) == ((16, 16) if few else (0, 32))
+        c.check_tolerance(c.run_plan(vb.Plan(c.matrix, rhs)), f"rhs={rhs}")
+        c.close()

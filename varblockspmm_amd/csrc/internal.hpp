@@ -126,6 +126,9 @@ struct HostSchedule {
   // on one workgroup, so the longest row must stay within kTileSpanLimit
   // times the mean steps per workgroup slot.
   bool rhs64_tiles{};
+  // Columns per workgroup of the split-k kernel at RHS 32 (0: all) and 64.
+  int32_t rhs32_columns{};
+  int32_t rhs64_columns{};
   HostSplitSchedule split;
   // Whether the split-row path pays off for this matrix at RHS 16 and up:
   // the row-owned launch would leave most CUs idle while its rows are long.

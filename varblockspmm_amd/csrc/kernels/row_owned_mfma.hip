@@ -4,16 +4,18 @@
 //
 // Work unit.  One workgroup (4 waves) owns one block row of height h and
 // writes its h x RHS slab of C, or owns up to four light rows, one per wave
-// (the schedule packs rows of at most kPackSteps k steps, kPackStepsRhs64 at
-// RHS 64); nothing else writes those slabs, so there are no atomics and no
-// global workspace.  A
+// (the schedule packs rows of at most kPackSteps k steps); nothing else writes
+// those slabs, so there are no atomics and no global workspace.  RHS is 8, 16
+// or 32 here: wider products, and RHS 32 products of few rows, give each
+// column part of a slab a workgroup of its own (blockIdx.y; the schedule's
+// columns rule), and the tile split (row_tiles_kernel) is RHS 64 in one.  A
 // row's k steps (16 columns of one block, or the 8 that end a block whose
 // width is 8 mod 16; one precomputed record each) are dealt to the waves
 // that share it -- four, in runs of two, or a packed row's one wave; each
 // wave accumulates all T = ceil(h/16) row tiles for its steps.  The four
 // partial slabs of a shared row are summed in LDS in a fixed order,
 // (w0 + w2) + (w1 + w3): at RHS 16 and 32 by wave 0 after one barrier, at
-// RHS 8 and 64 in pairs over three barriers.  A packed row's wave stores its
+// RHS 8 (and the VALU variant's 64) in pairs over three barriers.  A packed row's wave stores its
 // sums itself.  The accumulation order depends only on the matrix, so
 // results are bit-identical from run to run.
 //
@@ -69,6 +71,7 @@
 // MFMAs.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 
@@ -188,6 +191,7 @@ struct Launch {
   const float* b;
   float* c;
   int64_t ldc;  // C's leading dimension: scalar_rows, or a split-row workspace's virtual rows
+  int64_t part_b, part_c;  // floats from one column part's B and C to the next's (blockIdx.y takes a part)
 };
 
 // Fixed-order reduction of the four partial slabs of a shared row,
@@ -513,12 +517,18 @@ __device__ __forceinline__ void row_body(const Launch& L, const WaveItem& item, 
   }
 }
 
-template <int RHS, bool kValu, bool kWideB>
+// kParts: the workgroup computes column part blockIdx.y (an instantiation of
+// its own: the offsets cost 0.1 us of a 12 us product that has one part).
+template <int RHS, bool kValu, bool kWideB, bool kParts>
 __global__ __launch_bounds__(kThreads) void row_owned_mfma_kernel(Launch L) {
   __shared__ __attribute__((aligned(16))) char lds[Lds<RHS, kValu>::kTotal];
   const int wave = uniform(int(threadIdx.x) / kWave);
   const int lane = int(threadIdx.x) % kWave;
   const WaveItem item = L.items[int64_t(blockIdx.x) * kWaves + wave];
+  if constexpr (kParts) {
+    L.b += int64_t(blockIdx.y) * L.part_b;
+    L.c += int64_t(blockIdx.y) * L.part_c;
+  }
   // An idle wave leaves.  A workgroup whose row is shared has no idle wave,
   // so no wave that leaves here is awaited at a barrier.
   if (uniform(item.step_count) < 0) return;
@@ -682,39 +692,42 @@ __global__ __launch_bounds__(kThreads) void row_tiles_kernel(Launch L) {
   }
 }
 
-// tiles: RHS 64 runs the tile-split kernel (the MFMA kernel only).
+// RHS: the columns of one workgroup.  The MFMA kernel at 64 is the tile split.
 template <int RHS, bool kValu, bool kWideB>
-void launch(const Launch& L, int64_t groups, bool tiles, hipStream_t stream) {
-  if (RHS == 64 && !kValu && tiles)
+void launch(const Launch& L, int64_t groups, int parts, hipStream_t stream) {
+  if constexpr (RHS == 64 && !kValu)
     row_tiles_kernel<kWideB><<<dim3(unsigned(groups)), dim3(kThreads), 0, stream>>>(L);
+  else if ((RHS == 16 || RHS == 32) && !kValu && parts > 1)
+    row_owned_mfma_kernel<RHS, kValu, kWideB, (RHS == 16 || RHS == 32) && !kValu>
+        <<<dim3(unsigned(groups), unsigned(parts)), dim3(kThreads), 0, stream>>>(L);
   else
-    row_owned_mfma_kernel<RHS, kValu, kWideB><<<dim3(unsigned(groups)), dim3(kThreads), 0, stream>>>(L);
+    row_owned_mfma_kernel<RHS, kValu, kWideB, false><<<dim3(unsigned(groups)), dim3(kThreads), 0, stream>>>(L);
 }
 
 template <bool kValu, bool kWideB>
-void launch_rhs(const Launch& L, int64_t groups, int rhs, bool tiles, hipStream_t stream) {
-  switch (rhs) {
-  case 8: launch<8, kValu, kWideB>(L, groups, false, stream); break;
-  case 16: launch<16, kValu, kWideB>(L, groups, false, stream); break;
-  case 32: launch<32, kValu, kWideB>(L, groups, false, stream); break;
-  default: launch<64, kValu, kWideB>(L, groups, tiles, stream); break;
+void launch_columns(const Launch& L, int64_t groups, int columns, int parts, hipStream_t stream) {
+  switch (columns) {
+  case 8: launch<8, kValu, kWideB>(L, groups, parts, stream); break;
+  case 16: launch<16, kValu, kWideB>(L, groups, parts, stream); break;
+  case 32: launch<32, kValu, kWideB>(L, groups, parts, stream); break;
+  default: launch<64, kValu, kWideB>(L, groups, parts, stream); break;
   }
 }
 
 // wide: 64-bit B addressing (the MFMA kernel only; the VALU variant keeps
 // the 32-bit offset bound).
 template <bool kValu>
-void launch_items(const Launch& L, int64_t groups, int rhs, bool wide, bool tiles, hipStream_t stream) {
+void launch_items(const Launch& L, int64_t groups, int columns, int parts, bool wide, hipStream_t stream) {
   if (groups <= 0) return;
   if (groups > int64_t(0x7fffffff)) throw std::invalid_argument("schedule too large for one launch");
   if constexpr (kValu) {
     if (wide) throw std::invalid_argument("the VALU variant needs (min(rhs, 16) - 1) * K * 4 + 128 <= 0xfffffff0");
-    launch_rhs<true, false>(L, groups, rhs, false, stream);
+    launch_columns<true, false>(L, groups, columns, parts, stream);
   } else {
     if (wide)
-      launch_rhs<false, true>(L, groups, rhs, tiles, stream);
+      launch_columns<false, true>(L, groups, columns, parts, stream);
     else
-      launch_rhs<false, false>(L, groups, rhs, tiles, stream);
+      launch_columns<false, false>(L, groups, columns, parts, stream);
   }
   check_hip(hipGetLastError(), "row_owned_mfma launch");
 }
@@ -726,6 +739,13 @@ void launch_items(const Launch& L, int64_t groups, int rhs, bool wide, bool tile
 // C stores are contiguous; the loads of four parts are issued before their
 // adds, so a lane waits for memory once per four parts.
 constexpr int kReduceThreads = 256;
+
+// Columns of one workgroup of the partial launch: 16 up to this many
+// workgroups of the split schedule, 32 past it.  Measured at degree 16 (high
+// sizes), 16 / 32 columns against all 64 (or 32): 64 rows (320 workgroups)
+// RHS 64 10.4 / 10.7 / 12.4 us, RHS 32 8.7 / 9.1 us; 128 rows (640) RHS 64
+// 17.6 / 15.5 / 16.6 us.
+constexpr int64_t kSplitFewGroups = 384;
 
 __global__ __launch_bounds__(kReduceThreads) void split_reduce_kernel(const SplitRowRec* rows, const float* w,
                                                                       int64_t ldw, float* c, int64_t ldc, int rhs) {
@@ -791,15 +811,21 @@ void launch_row_owned_math(const vbsr_device_view& a, const vbsr_row_schedule& s
                            bool wide_b, hipStream_t stream) {
   if (!supported_rhs(rhs)) throw std::invalid_argument("unsupported rhs width");
   check_panels(a, b, c, rhs);
-  const void* rows = rhs >= 32 && s.rows_wide != nullptr ? s.rows_wide : s.rows;
+  // The columns of one workgroup: at RHS 64 the MFMA kernel is the tile split
+  // over all of them (rhs64_tiles) or the split-k kernel over 16 or 32; at
+  // RHS 32 the split-k kernel may take 16 at a time.
+  int columns = rhs;
+  if (!kValu && (rhs == 32 || (rhs == 64 && s.rhs64_tiles == 0))) {
+    const int32_t part = rhs == 32 ? s.rhs32_columns : s.rhs64_columns;
+    if (part != 0 && part != 16 && part != 32)
+      throw std::invalid_argument("schedule's columns per workgroup must be 0, 16 or 32");
+    columns = part != 0 ? part : 32;
+  }
+  const void* rows = columns >= 32 && s.rows_wide != nullptr ? s.rows_wide : s.rows;
   int64_t groups = s.groups;
-  const bool tiles = !kValu && rhs == 64 && s.rhs64_tiles != 0;
-  if (tiles) {
-    rows = s.rows_tile;
-    groups = s.groups_tile;
-  } else if (rhs == 64 && s.rows_rhs64 != nullptr) {
-    rows = s.rows_rhs64;
-    groups = s.groups_rhs64;
+  if (columns == 64) {
+    rows = kValu ? s.rows_rhs64 : s.rows_tile;
+    groups = kValu ? s.groups_rhs64 : s.groups_tile;
   }
   // A matrix with block rows has at least one workgroup in every order (empty
   // rows included), so a schedule whose chosen order is missing or empty
@@ -808,10 +834,8 @@ void launch_row_owned_math(const vbsr_device_view& a, const vbsr_row_schedule& s
   if (a.block_rows > 0 && (rows == nullptr || groups <= 0 || s.steps == nullptr))
     throw std::invalid_argument("schedule has no launch order for this matrix (take it from vbsr_matrix_row_schedule)");
   const Launch L{a, static_cast<const StepRec*>(s.steps), static_cast<const WaveItem*>(rows), s.step_limit, b, c,
-                 a.scalar_rows};
-  // At RHS 64 the schedule says which kernel runs: the split-k kernel or
-  // the tile split (rhs64_tiles, set by the matrix's rule).
-  launch_items<kValu>(L, groups, rhs, wide_b || !narrow_b_offsets(a, rhs), tiles, stream);
+                 a.scalar_rows, columns * a.scalar_cols, columns * a.scalar_rows};
+  launch_items<kValu>(L, groups, columns, rhs / columns, wide_b || !narrow_b_offsets(a, columns), stream);
 }
 
 }  // namespace
@@ -847,9 +871,10 @@ void launch_split_row(const vbsr_device_view& a, const vbsr_row_schedule& s, con
     check_panels(split.virtual_rows, a.scalar_rows, c, workspace, rhs);
   }
   if (a.block_rows <= 0) return;
+  const int columns = std::min(rhs, split.groups <= kSplitFewGroups ? 16 : 32);
   const Launch L{a, static_cast<const StepRec*>(s.steps), split.items, s.step_limit, b, workspace,
-                 split.virtual_rows};
-  launch_items<false>(L, split.groups, rhs, !narrow_b_offsets(a, rhs), false, stream);
+                 split.virtual_rows, columns * a.scalar_cols, columns * split.virtual_rows};
+  launch_items<false>(L, split.groups, columns, rhs / columns, !narrow_b_offsets(a, columns), stream);
   // A row's slab holds at most 64 * rhs elements.
   const unsigned chunks = unsigned((64 * rhs + kReduceThreads - 1) / kReduceThreads);
   split_reduce_kernel<<<dim3(unsigned(a.block_rows), chunks), dim3(kReduceThreads), 0, stream>>>(

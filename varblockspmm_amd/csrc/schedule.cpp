@@ -271,6 +271,27 @@ HostSchedule build_schedule(const vbsr_host_view& m) {
     out.rhs64_tiles = rows > 0 && longest * kTileSlots <= kTileSpanLimit * total;
   }
 
+  // Columns per workgroup of the split-k kernel.  A workgroup reads at most
+  // about 90 GB/s, so few workgroups leave most of the card's rate unused:
+  // taking 16 columns at a time at RHS 32 and 64 gives two and four times the
+  // workgroups for reading A again, from L2 for the most part.  Measured (high
+  // sizes, random columns, calls back to back), 16 columns against 32 at
+  // RHS 32, and 16 / 32 against all 64 at RHS 64:
+  //   64 rows of degree 16    8.3 / 11.6 us    9.2 / 11.6 / 18.4 us
+  //   128 rows of degree 16   8.8 / 11.5 us   13.8 / 13.8 / 20.5 us
+  //   203 rows of degree 8    8.0 /  8.6 us   11.7 / 11.7 / 13.5 us
+  //   203 rows of degree 16  12.4 / 12.1 us   19.7 / 18.2 / 20.2 us
+  //   512 rows of degree 2    6.2 /  6.8 us    8.6 /  9.0 / 14.0 us
+  //   512 rows of degree 8   14.2 / 12.7 us   22.3 / 18.4 / 19.8 us
+  // All 64 columns in one workgroup took 96 + 64 registers and was within 3%
+  // of 32 at best, so at RHS 64 the split-k kernel takes 16 or 32.
+  {
+    constexpr size_t kFewUnits = 128, kSomeUnits = 384, kSomeSteps = 4096;
+    const bool few = n_units <= kFewUnits || (n_units <= kSomeUnits && out.steps.size() <= kSomeSteps);
+    out.rhs32_columns = few ? 16 : 0;
+    out.rhs64_columns = few ? 16 : 32;
+  }
+
   // Split-row schedule.  Parts of a row hold part_steps consecutive steps (a
   // multiple of one run per wave, sized so that the parts of the whole
   // matrix fill about kSplitTargetGroups workgroups); the row's last part
