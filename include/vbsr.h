@@ -174,6 +174,8 @@ typedef struct vbsr_row_schedule {
    * workgroups.  Set by the matrix's rule, 16 where rows are few; a caller may
    * set either value in its copy of the struct. */
   int32_t rhs32_columns, rhs64_columns;
+  const void* steps_tile;  /* device: one 16-byte record per step of the tile split */
+  int32_t step_limit_tile; /* index of its last one */
 } vbsr_row_schedule;
 int vbsr_matrix_row_schedule(const vbsr_matrix* matrix, vbsr_row_schedule* out);
 

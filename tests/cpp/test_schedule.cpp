@@ -18,6 +18,8 @@
 //   * the split-row schedule: each row's parts cover its steps in order and
 //     take consecutive virtual rows, every part is in exactly one workgroup,
 //     and the automatic choice follows its rule;
+//   * the tile split's steps cover each row's 8-column pieces in order, runs
+//     that are contiguous in B cut at kTileK columns;
 //   * building twice gives the same schedule;
 //   * matrices whose rows share few block columns (every row on the same 8
 //     columns; rows overlapping in 15 of 16 columns) build in seconds: the
@@ -31,6 +33,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <utility>
 #include <vector>
 
 #include "internal.hpp"
@@ -269,6 +272,44 @@ bool same(const std::vector<vbsr_amd::WaveItem>& a, const std::vector<vbsr_amd::
   return a.size() == b.size() && (a.empty() || std::memcmp(a.data(), b.data(), a.size() * sizeof(a[0])) == 0);
 }
 
+// The tile split's steps: each row's, expanded to 8-column pieces, are the
+// row's blocks' pieces in order, with their A and B offsets; a step is 1 to 4
+// pieces, and is cut short only where the next piece is not contiguous in B.
+// The device's tile items count them and are rows_tile otherwise.
+void check_tile_steps(const vbsr_host_view& m, const vbsr_amd::HostSchedule& s) {
+  using vbsr_amd::kTileOffsetMask;
+  using vbsr_amd::kTilePieceShift;
+  constexpr int64_t kMost = vbsr_amd::kTileK / 8;
+  CHECK(s.tile_first.size() == size_t(m.block_rows) + 1 && s.tile_first[0] == 0);
+  CHECK(size_t(s.tile_first[size_t(m.block_rows)]) == s.steps_tile.size());
+  for (int32_t i = 0; i < m.block_rows; ++i) {
+    std::vector<std::pair<int64_t, int64_t>> got, want;
+    int64_t last_pieces = kMost;
+    for (int32_t q = s.tile_first[size_t(i)]; q < s.tile_first[size_t(i) + 1]; ++q) {
+      const auto& step = s.steps_tile[size_t(q)];
+      const int64_t b = step.b_off & kTileOffsetMask, pieces = (step.b_off >> kTilePieceShift) + 1;
+      CHECK(pieces >= 1 && pieces <= kMost);
+      CHECK(last_pieces == kMost || got.back().second + 8 != b);
+      for (int64_t p = 0; p < pieces; ++p) got.emplace_back(step.a_off + 8 * p * m.row_size[i], b + 8 * p);
+      last_pieces = pieces;
+    }
+    for (int32_t blk = m.row_ptr[i]; blk < m.row_ptr[i + 1]; ++blk)
+      for (int32_t k = 0; k < m.col_size[m.block_col[blk]]; k += 8)
+        want.emplace_back(m.value_off[blk] + int64_t(k) * m.row_size[i], m.col_scalar_off[m.block_col[blk]] + k);
+    CHECK(got == want);
+  }
+  const std::vector<vbsr_amd::WaveItem> items = s.tile_items();
+  CHECK(items.size() == s.rows_tile.size());
+  for (size_t q = 0; q < items.size(); ++q) {
+    const int32_t i = s.rows_tile[q].row;
+    CHECK(items[q].row == i && items[q].c_off == s.rows_tile[q].c_off && items[q].h == s.rows_tile[q].h);
+    CHECK((items[q].step_count < 0) == (s.rows_tile[q].step_count < 0) && items[q].group == s.rows_tile[q].group);
+    if (i < 0) continue;
+    CHECK(items[q].step_first == s.tile_first[size_t(i)]);
+    CHECK(items[q].step_count == s.tile_first[size_t(i) + 1] - s.tile_first[size_t(i)]);
+  }
+}
+
 // reorders: the matrix is random enough that a chained order must differ
 // from the heaviest-first one.
 void check_view(const vbsr_host_view& m, const char* name, double max_seconds, bool reorders = false) {
@@ -282,6 +323,7 @@ void check_view(const vbsr_host_view& m, const char* name, double max_seconds, b
   }
   check_steps(m, s);
   check_split(m, s);
+  check_tile_steps(m, s);
   CHECK(s.rhs64_tiles == expected_tiles(m));
   std::vector<int> xcd_of_row(size_t(m.block_rows), -1);
   check_order(m, s, s.rows, xcd_of_row, false, s.groups, vbsr_amd::kPackSteps);

@@ -102,3 +102,30 @@ def test_few_rows_take_their_columns_in_parts(rows, degree, few):
         assert (schedule.rhs32_columns, schedule.rhs64_columns) == ((16, 16) if few else (0, 32))
         c.check_tolerance(c.run_plan(vb.Plan(c.matrix, rhs)), f"rhs={rhs}")
         c.close()
+
+
+# Runs of block columns that are contiguous in B, of 8 to 72 columns, beside others that are not: the tile split's
+# steps hold 1 to 4 pieces of 8 columns and cross blocks; block column 7 (NaN below) is in no row.
+TILE_WIDTHS = [8, 8, 24, 16, 8, 40, 64, 16, 8, 56, 8]
+TILE_ROWS = [[0], [0, 1], [0, 1, 2], [1, 2, 3], [0, 1, 2, 3, 4], [4, 5], [5, 6], [2, 0, 1, 10], [8, 9, 10], [9], [],
+             [6, 5, 4, 3, 2, 1, 0], [3, 3, 4, 4], list(range(7)) + [8, 9, 10]]
+
+
+@pytest.mark.parametrize("h", range(8, 65, 8))
+def test_tile_split_steps_across_blocks(h):
+    """RHS 64's tile split with every row of height h, and of h beside the next heights: within tolerance of the
+    oracle, both forms of B's addressing bit-identical, and rows of B that no block names never read into a sum."""
+    parity.note(f"tile steps h={h}")
+    host = parity.hand_made([8 * (1 + (h // 8 - 1 + i * (i % 2)) % 8) for i in range(len(TILE_ROWS))], TILE_WIDTHS,
+                            TILE_ROWS, seed=h)
+    c = parity.Case(host, 64, 41)
+    view, schedule = c.matrix.device_view(), c.matrix.row_schedule()
+    schedule.rhs64_tiles = 1
+    b = c.b.reshape(64, host.scalar_cols).copy()
+    b[:, host.col_scalar_off[7]:host.col_scalar_off[8]] = np.nan
+    c.b_dev = torch.from_numpy(b.reshape(-1)).to(parity.DEVICE)
+    first = c.run(lambda: vb.launch_row_owned(view, schedule, c.b_dev, c.c_dev, 64, c.stream))
+    c.check_tolerance(first, f"h={h}")
+    wide = c.run(lambda: vb.launch_row_owned_wide_b(view, schedule, c.b_dev, c.c_dev, 64, c.stream))
+    np.testing.assert_array_equal(bits(wide), bits(first))
+    c.close()

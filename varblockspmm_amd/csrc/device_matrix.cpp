@@ -61,7 +61,10 @@ DeviceMatrix::DeviceMatrix(const vbsr_host_view& host) {
     schedule_.groups = schedule.groups;
     schedule_.rows_rhs64 = upload(schedule.rows_rhs64.data(), int64_t(schedule.rows_rhs64.size()), allocations_);
     schedule_.groups_rhs64 = schedule.groups_rhs64;
-    schedule_.rows_tile = upload(schedule.rows_tile.data(), int64_t(schedule.rows_tile.size()), allocations_);
+    const std::vector<WaveItem> tile_items = schedule.tile_items();
+    schedule_.rows_tile = upload(tile_items.data(), int64_t(tile_items.size()), allocations_);
+    schedule_.steps_tile = upload(schedule.steps_tile.data(), int64_t(schedule.steps_tile.size()), allocations_);
+    schedule_.step_limit_tile = int32_t(std::max<size_t>(schedule.steps_tile.size(), 1) - 1);
     schedule_.groups_tile = schedule.groups_tile;
     schedule_.rhs64_tiles = schedule.rhs64_tiles ? 1 : 0;
     schedule_.rhs32_columns = schedule.rhs32_columns;

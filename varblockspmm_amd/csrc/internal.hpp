@@ -54,6 +54,13 @@ struct alignas(16) StepRec {
 static_assert(sizeof(StepRec) == 16, "StepRec is read as one dwordx4");
 constexpr int64_t kHalfStep = int64_t(1) << 62;
 
+// A step of the RHS 64 tile split: up to kTileK columns that are contiguous
+// in B (and, like all of a row's columns, in A).  a_off as above; b_off holds
+// the first B row and, from kTilePieceShift up, its 8-column pieces less one.
+constexpr int kTileK = 32;
+constexpr int kTilePieceShift = 60;
+constexpr int64_t kTileOffsetMask = (int64_t(1) << kTilePieceShift) - 1;
+
 // The row-owned kernel's workgroup: kRowWaves waves.  They hold either one
 // block row together -- its k steps dealt to the waves in runs of kStepRun
 // consecutive steps (wave w's first step is the row's step kStepRun * w) and
@@ -121,6 +128,11 @@ struct HostSchedule {
   // chained like the other orders.
   std::vector<WaveItem> rows_tile;
   int64_t groups_tile{};
+  // The tile split's steps, and each block row's first (block_rows + 1).  The
+  // device's tile items count these steps (tile_items).
+  std::vector<StepRec> steps_tile;
+  std::vector<int32_t> tile_first;
+  std::vector<WaveItem> tile_items() const;
   // Whether RHS 64 runs the tile-split kernel over rows_tile instead of the
   // split-k kernel over rows_rhs64: a row's steps then run one after another
   // on one workgroup, so the longest row must stay within kTileSpanLimit

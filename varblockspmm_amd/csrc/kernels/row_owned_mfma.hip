@@ -81,6 +81,7 @@ namespace vbsr_amd {
 namespace {
 
 using f32x4 = float __attribute__((ext_vector_type(4)));
+using f32x2 = float __attribute__((ext_vector_type(2)));
 // The same vector at float alignment: B and C panels need only be 4-byte
 // aligned.  gfx950 serves 16-byte global and buffer accesses at any 4-byte
 // aligned address (ROCm runs it in unaligned access mode, and the compiler
@@ -544,24 +545,50 @@ __global__ __launch_bounds__(kThreads) void row_owned_mfma_kernel(Launch L) {
 // (the schedule's tile order gives every row with k steps a workgroup of its
 // own and packs only empty rows, four to a workgroup, which it takes one
 // after another), and all four waves work on it: wave w computes RHS tile w
-// (C columns 16 w .. 16 w + 15) over all of the row's k steps, in step
-// order.
-// A step's A tile (16 block columns, 64 h bytes) is loaded once for the
-// workgroup, 16 bytes per lane, into one of two LDS buffers, and one barrier
-// per step publishes it; each wave moves its own B tile through its own LDS
-// slot.  There is no cross-wave reduction, and a wave holds T row tiles of
-// one RHS tile: a quarter of the split-k kernel's accumulators, so a SIMD
-// holds 6 of these waves against 3 of the split-k kernel's.  The price is
-// that a row's steps run one after another on one workgroup, so the launch
-// is as long as its longest row; the schedule takes this kernel only where
-// that stays short against the work per workgroup slot (rhs64_tiles).
-constexpr int kTileLd = 16 * kMaxTiles + 4;  // A buffer: float (r, k) at k * kTileLd + r
-constexpr int kTileFloats = 16 * kTileLd;
-constexpr int kTileLdsBytes = 2 * kTileFloats * 4 + kWaves * kWave * 16;
+// (C columns 16 w .. 16 w + 15) over all of the row's columns, in order.
+//
+// A tile step is up to kTileK = 32 columns: a run of block columns of the row
+// that are contiguous in B (one block's, or those of blocks in adjacent
+// block columns), cut at 32; its last piece is 8, 16 or 24 wide.  Its A tile
+// (contiguous, up to 8 KB) is loaded once for the workgroup, 16 bytes per
+// lane and load, into one of two LDS buffers, and one barrier per step
+// publishes it; each wave moves its own B tile, eight lanes to a column, so
+// that a column's 128 bytes are read at once, through its own LDS slot.
+// There is no cross-wave reduction.
+//
+// What bounds it: L2's rate to the CUs where rows share block columns (every
+// piece of a B column that a step reads costs the one or two 128-byte lines
+// that it touches), L2 misses where they do not.  Against steps of 16 columns
+// of one block, half of them half empty: L2 reads 2.5e7 -> 2.0e7 lines and
+// 253 -> 225 us at 8192 block rows of degree 16 (low sizes, clamped columns),
+// 59.4 -> 55.0 us at 4096 rows of degree 8 (32 x 32 blocks, local), 90.0 ->
+// 87.6 us with high sizes and random columns, 166 -> 163 us at degree 16 with
+// sizes 8 or 64 (7.2 TB/s of L2 misses).  Lanes past a step's columns must
+// read nothing: letting them read on cost 12% there.  With the 16-column
+// steps, 14% fewer MFMAs, 5 waves per SIMD instead of 6, and three or four
+// register stages each changed nothing.
+// The price of one workgroup per row is that a row's steps run one after
+// another, so the launch is as long as its longest row; the schedule takes
+// this kernel only where that stays short against the work per workgroup
+// slot (rhs64_tiles).
+constexpr int kTileLd = 16 * kMaxTiles + 8;  // A buffer: float (r, k) at k * kTileLd + r; 2 kTileLd is 16 mod 64
+constexpr int kTileFloats = kTileK * kTileLd;
+constexpr int kTileSlot = 16 * kTileK;  // floats of a wave's B slot
+constexpr int kTileLdsBytes = (2 * kTileFloats + kWaves * kTileSlot) * 4;
+
+// Float k of column n of a wave's B slot: column-major, a column's eight
+// 16-byte pieces permuted by an XOR of n's upper bits, so that the writes
+// (eight lanes to a column) and the reads (16 columns of one piece) cover all
+// banks.
+__device__ __forceinline__ int tile_slot_index(int n, int k) {
+  return n * kTileK + ((((k >> 2) ^ (n >> 1)) & 7) << 2) + (k & 3);
+}
 
 template <int T, bool kWideB>
 __device__ __forceinline__ void tile_row(const Launch& L, const WaveItem& item, char* lds, int wave, int lane) {
   constexpr int ld = kTileLd;
+  // A loads of a step: kThreads threads of 16 bytes cover 1024 floats.
+  constexpr int kALoads = (16 * T * kTileK + 4 * kThreads - 1) / (4 * kThreads);
   const int tid = wave * kWave + lane;
   const int group = lane >> 4;
   const int x = lane & 15;
@@ -571,80 +598,104 @@ __device__ __forceinline__ void tile_row(const Launch& L, const WaveItem& item, 
   const int last_rows = h - 16 * (T - 1);
   const uint32_t ldb = uint32_t(L.a.scalar_cols);
   float* a_bufs = reinterpret_cast<float*>(lds);
-  f32x4* b_slot = reinterpret_cast<f32x4*>(lds + 2 * kTileFloats * 4) + wave * kWave;
+  float* b_slot = reinterpret_cast<float*>(lds) + 2 * kTileFloats + wave * kTileSlot;
 
-  // This thread's 16 bytes of the step's column-major h x 16 A tile go to
-  // float (k, r) of the buffer (f / h computed as in row_body); threads past
-  // the tile hold zeros and write them to the never-read padding rows.
-  const uint32_t h_recip = uint32_t(uniform(int((65536u + uint32_t(h) - 1u) / uint32_t(h))));
-  const int f = 4 * tid;
-  const int fk = int((uint32_t(f) * h_recip) >> 16);
-  const int a_write = f < 16 * h ? fk * ld + (f - fk * h) : (tid & 15) * ld + 16 * kMaxTiles;
-  const int a_read = 4 * group * ld + x;
-  const int a_read_last = 4 * group * ld + 16 * (T - 1) + (x & (last_rows - 1));
-  const uint32_t a_full_bytes = uint32_t(16 * h) * 4u;
-  const uint32_t a_half_bytes = uint32_t(8 * h) * 4u;
+  // This thread's 16 bytes of load q of the step's column-major A tile go to
+  // float (k, r) of the buffer; f / h is (f * ceil(2^20 / h)) >> 20, exact for
+  // f < 2048 and h up to 64.  Threads past h x 32 hold zeros and write them to
+  // the never-read padding rows.
+  const uint32_t h_recip = uint32_t(uniform(int(((1u << 20) + uint32_t(h) - 1u) / uint32_t(h))));
+  int a_write[kALoads];
+#pragma unroll
+  for (int q = 0; q < kALoads; ++q) {
+    const int f = 4 * kThreads * q + 4 * tid;
+    const int fk = int((uint32_t(f) * h_recip) >> 20);
+    a_write[q] = f < kTileK * h ? fk * ld + (f - fk * h) : (tid & (kTileK - 1)) * ld + 16 * kMaxTiles;
+  }
+  // MFMAs 2 p and 2 p + 1 of a step take k = 8 p + 2 g + i, i = 0, 1, from
+  // lane group g; p runs over the step's 8-column pieces.
+  const int a_read = 2 * group * ld + x;
+  const int a_read_last = 2 * group * ld + 16 * (T - 1) + (x & (last_rows - 1));
 
-  // B: lane 4n + q of wave w reads B[k0 + 4q .. k0 + 4q + 3, 16 w + n], as
-  // one tile of the split-k kernel.
-  const int b_n = lane >> 2;
-  const int b_q = lane & 3;
-  const uint32_t b_full = uint32_t(b_n) * ldb * 4u + uint32_t(16 * b_q);
-  const uint32_t b_half = b_q < 2 ? b_full : kOutOfRange;
-  const uint32_t b_span = 15u * ldb * 4u;
-  const int64_t b_lane = int64_t(b_n) * L.a.scalar_cols + 4 * b_q;  // kWideB: the lane's float offset
-  const int slot_write = b_slot_index(b_n, b_q);
-  const int slot_read = b_slot_index(x, group);
+  // B: lane 8 n + q of wave w reads B[k0 + 4 q .. k0 + 4 q + 3, 16 w + n] and
+  // the same of column 16 w + 8 + n.
+  const int b_n = lane >> 3;
+  const int b_k = (lane & 7) * 4;
+  const uint32_t b_lane_bytes = uint32_t(b_n) * ldb * 4u + uint32_t(4 * b_k);
+  const uint32_t b_span = 7u * ldb * 4u;
+  const int64_t b_lane = int64_t(b_n) * L.a.scalar_cols + b_k;  // kWideB: the lane's float offset
+  const int b_write[2] = {tile_slot_index(b_n, b_k), tile_slot_index(8 + b_n, b_k)};
+  int b_read[kTileK / 8];
+#pragma unroll
+  for (int p = 0; p < kTileK / 8; ++p) b_read[p] = tile_slot_index(x, 8 * p + 2 * group);
 
   f32x4 acc[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   struct TileStage {
-    f32x4 a, b;
+    f32x4 a[kALoads];
+    f32x4 b[2];
+    int pieces;  // of eight columns; 0 past the segment
   };
   int parity = 0;  // A buffer of the next step
   for (int seg = 0; seg < count; seg += kWave) {
     const int seg_count = min(kWave, count - seg);
     const StepRec rec = L.steps[min(first + seg + min(lane, seg_count - 1), L.step_limit)];
     auto issue = [&](TileStage& st, int j) {
-      const bool live = j < seg_count;
       const int l = min(j, kWave - 1);
       const int64_t a_off = lane_value(rec.a_off, l);
       const int64_t b_word = lane_value(rec.b_off, l);
-      const bool half = (b_word & kHalfStep) != 0;
-      const rsrc_t a_rsrc = make_rsrc(L.a.values + a_off, live ? (half ? a_half_bytes : a_full_bytes) : 0u);
-      st.a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, 16 * tid, 0, kNonTemporal));
-      const float* b_base = L.b + (b_word & kOffsetMask) + int64_t(wave) * 16 * L.a.scalar_cols;
-      if constexpr (kWideB) {
-        st.b = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (live && (!half || b_q < 2)) st.b = *reinterpret_cast<const f32x4_unaligned*>(b_base + b_lane);
-      } else {
-        const rsrc_t b_rsrc = make_rsrc(b_base, live ? b_span + (half ? 32u : 64u) : 0u);
-        st.b = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, int(half ? b_half : b_full), 0, 0));
+      st.pieces = j < seg_count ? int(b_word >> kTilePieceShift) + 1 : 0;
+      const uint32_t k_bytes = uint32_t(st.pieces) * 32u;
+      const rsrc_t a_rsrc = make_rsrc(L.a.values + a_off, k_bytes * uint32_t(h));
+#pragma unroll
+      for (int q = 0; q < kALoads; ++q)
+        st.a[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                a_rsrc, 16 * tid + 16 * kThreads * q, 0, kNonTemporal));
+      const float* b_base = L.b + (b_word & kTileOffsetMask) + int64_t(wave) * 16 * L.a.scalar_cols;
+      const bool take = b_k < 8 * st.pieces;  // lanes past the step's k read nothing: they would touch more lines
+      const uint32_t b_bytes = take ? b_lane_bytes : kOutOfRange;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const float* base = b_base + int64_t(q) * 8 * L.a.scalar_cols;
+        if constexpr (kWideB) {
+          st.b[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+          if (take) st.b[q] = *reinterpret_cast<const f32x4_unaligned*>(base + b_lane);
+        } else {
+          const rsrc_t b_rsrc = make_rsrc(base, b_span + k_bytes);
+          st.b[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, int(b_bytes), 0, 0));
+        }
       }
     };
-    // Writes the step's A quarter and B tile, publishes the A tile with one
-    // barrier, runs the wave's T x 4 MFMAs.  The two A buffers alternate: a
-    // wave writes buffer p only after the barrier of the step before, which
-    // every wave reaches after its reads of buffer p two steps back.
+    // Writes the step's A share and B tile, publishes the A tile with one
+    // barrier, runs the wave's T x 2 MFMAs per piece.  The two A buffers
+    // alternate: a wave writes buffer p only after the barrier of the step
+    // before, which every wave reaches after its reads of buffer p two steps
+    // back.
     auto compute = [&](const TileStage& st) {
       float* a = a_bufs + parity * kTileFloats;
       parity ^= 1;
-      *reinterpret_cast<f32x4*>(a + a_write) = st.a;
-      b_slot[slot_write] = st.b;
+#pragma unroll
+      for (int q = 0; q < kALoads; ++q) *reinterpret_cast<f32x4*>(a + a_write[q]) = st.a[q];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) *reinterpret_cast<f32x4*>(b_slot + b_write[q]) = st.b[q];
       __syncthreads();
-      const f32x4 bv = b_slot[slot_read];
 #pragma unroll
-      for (int t = 0; t < T; ++t)
+      for (int p = 0; p < kTileK / 8; ++p) {
+        if (p < st.pieces) {
+          const f32x2 bv = *reinterpret_cast<const f32x2*>(b_slot + b_read[p]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float av = t < T - 1 ? a[a_read + 16 * t + i * ld] : a[a_read_last + i * ld];
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[i], av, acc[t], 0, 0, 0);
+          for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              const float av = a[(t < T - 1 ? a_read + 16 * t : a_read_last) + (8 * p + i) * ld];
+              acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[i], av, acc[t], 0, 0, 0);
+            }
         }
+      }
     };
-    // Two stages, as in row_body: step j + 1 loads while step j computes; an
-    // odd count ends on a dead step (zero-byte loads, zeros multiplied in).
+    // Two stages, as in row_body: step j + 1 loads while step j computes.
     TileStage r0, r1;
     issue(r0, 0);
     for (int j = 0; j < seg_count; j += 2) {
@@ -653,7 +704,7 @@ __device__ __forceinline__ void tile_row(const Launch& L, const WaveItem& item, 
       compute(r0);
       issue(r0, j + 2);
       __builtin_amdgcn_sched_barrier(0);
-      compute(r1);
+      if (r1.pieces != 0) compute(r1);
     }
   }
   // Every wave's reads of this row's A buffers end before the next row of
@@ -823,17 +874,24 @@ void launch_row_owned_math(const vbsr_device_view& a, const vbsr_row_schedule& s
   }
   const void* rows = columns >= 32 && s.rows_wide != nullptr ? s.rows_wide : s.rows;
   int64_t groups = s.groups;
-  if (columns == 64) {
-    rows = kValu ? s.rows_rhs64 : s.rows_tile;
-    groups = kValu ? s.groups_rhs64 : s.groups_tile;
+  const void* steps = s.steps;
+  int32_t step_limit = s.step_limit;
+  if (columns == 64 && kValu) {
+    rows = s.rows_rhs64;
+    groups = s.groups_rhs64;
+  } else if (columns == 64) {
+    rows = s.rows_tile;
+    groups = s.groups_tile;
+    steps = s.steps_tile;
+    step_limit = s.step_limit_tile;
   }
   // A matrix with block rows has at least one workgroup in every order (empty
   // rows included), so a schedule whose chosen order is missing or empty
   // belongs to no matrix with rows: refuse it rather than launch nothing or
   // read through a null pointer.
-  if (a.block_rows > 0 && (rows == nullptr || groups <= 0 || s.steps == nullptr))
+  if (a.block_rows > 0 && (rows == nullptr || groups <= 0 || steps == nullptr))
     throw std::invalid_argument("schedule has no launch order for this matrix (take it from vbsr_matrix_row_schedule)");
-  const Launch L{a, static_cast<const StepRec*>(s.steps), static_cast<const WaveItem*>(rows), s.step_limit, b, c,
+  const Launch L{a, static_cast<const StepRec*>(steps), static_cast<const WaveItem*>(rows), step_limit, b, c,
                  a.scalar_rows, columns * a.scalar_cols, columns * a.scalar_rows};
   launch_items<kValu>(L, groups, columns, rhs / columns, wide_b || !narrow_b_offsets(a, columns), stream);
 }

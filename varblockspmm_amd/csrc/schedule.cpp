@@ -253,6 +253,28 @@ HostSchedule build_schedule(const vbsr_host_view& m) {
   // a workgroup of its own.
   out.groups_tile = launch_orders(0, nullptr, &out.rows_tile, nullptr);
 
+  // The tile split's steps: runs of a row's columns that are contiguous in B,
+  // cut at kTileK columns.  They are no more than the row's k steps.
+  out.tile_first.assign(static_cast<size_t>(rows) + 1, 0);
+  for (int32_t i = 0; i < rows; ++i) {
+    int64_t next_b = -1, pieces = 0;  // where the last step would go on, and its 8-column pieces
+    for (int32_t blk = m.row_ptr[i]; blk < m.row_ptr[i + 1]; ++blk) {
+      const int32_t col = m.block_col[blk];
+      for (int32_t k0 = 0; k0 < m.col_size[col]; k0 += 8) {
+        const int64_t b_off = m.col_scalar_off[col] + k0;
+        if (b_off != next_b || pieces == kTileK / 8) {
+          out.steps_tile.push_back({m.value_off[blk] + int64_t(k0) * m.row_size[i], b_off});
+          pieces = 0;
+        } else {
+          out.steps_tile.back().b_off += int64_t(1) << kTilePieceShift;
+        }
+        ++pieces;
+        next_b = b_off + 8;
+      }
+    }
+    out.tile_first[size_t(i) + 1] = int32_t(out.steps_tile.size());
+  }
+
   // RHS 64 kernel choice.  The tile-split kernel runs a row's steps one after
   // another on one workgroup (all four waves on each step), so its launch
   // lasts at least the longest row's steps.  It is taken when those stay
@@ -382,6 +404,16 @@ HostSchedule build_schedule(const vbsr_host_view& m) {
   for (int32_t i = 0; i < rows; ++i) longest = std::max(longest, steps_of(i));
   out.split_preferred = n_units < kSplitBelowGroups && longest > 2 * kRunSteps;
   return out;
+}
+
+std::vector<WaveItem> HostSchedule::tile_items() const {
+  std::vector<WaveItem> items = rows_tile;
+  for (WaveItem& item : items)
+    if (item.row >= 0) {
+      item.step_first = tile_first[size_t(item.row)];
+      item.step_count = tile_first[size_t(item.row) + 1] - item.step_first;
+    }
+  return items;
 }
 
 }  // namespace vbsr_amd
