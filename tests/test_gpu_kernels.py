@@ -129,3 +129,79 @@ def test_tile_split_steps_across_blocks(h):
     wide = c.run(lambda: vb.launch_row_owned_wide_b(view, schedule, c.b_dev, c.c_dev, 64, c.stream))
     np.testing.assert_array_equal(bits(wide), bits(first))
     c.close()
+
+
+def skewed(light, heavy, blocks, seed=0):
+    """`light` block rows of 0 to 2 blocks with rows of `blocks` blocks among them, of every height in turn."""
+    rows = []
+    for q in range(light + heavy):
+        is_heavy = (q + 1) * heavy // (light + heavy) != q * heavy // (light + heavy)
+        rows.append([(q + j) % 211 for j in range(blocks if is_heavy else q % 3)])
+    return parity.hand_made([8 * (1 + (5 * q) % 8) for q in range(len(rows))], [8 * (1 + (3 * j) % 8) for j in range(211)],
+                            rows, seed=seed)
+
+
+# (light rows, heavy rows, blocks of one) on both sides of the rule: 150 blocks are about 400 k steps
+SKEWED = {"one": (60, 1, 150, True), "many-heights": (700, 16, 150, True), "few-light-rows": (40, 9, 120, True),
+          "no-light-rows": (2, 9, 120, False), "not-long": (60, 1, 40, False)}
+
+
+@pytest.mark.parametrize("rhs", [8, 16, 32, 64])
+@pytest.mark.parametrize("name", list(SKEWED))
+def test_long_rows_split_over_workgroups(name, rhs):
+    """A plan whose long rows are split: three kernels, every output written (C starts as NaN, and holds the parts'
+    slabs meanwhile), within tolerance of the oracle, the same bits again, from launch_row_owned and with B's other
+    addressing; and within tolerance with the rows whole (long_count 0)."""
+    light, heavy, blocks, split = SKEWED[name]
+    parity.note(f"long rows {name} rhs={rhs}")
+    c = parity.Case(skewed(light, heavy, blocks, rhs), rhs, 43)
+    view, schedule = c.matrix.device_view(), c.matrix.row_schedule()
+    schedule.long_rhs64 = 1
+    assert (schedule.long_count > 0) == split
+    plan = vb.Plan(c.matrix, rhs)
+    splits = split and not (rhs == 64 and (schedule.rhs64_tiles or not c.matrix.row_schedule().long_rhs64))
+    assert plan.launch_count() == (3 if splits else 1)
+    planned = c.run_plan(plan)
+    c.check_tolerance(planned, f"{name} plan")
+    np.testing.assert_array_equal(bits(c.run_plan(plan)), bits(planned))
+    schedule.rhs64_tiles = 0
+    first = c.run(lambda: vb.launch_row_owned(view, schedule, c.b_dev, c.c_dev, rhs, c.stream))
+    c.check_tolerance(first, f"{name} split")
+    if splits:
+        np.testing.assert_array_equal(bits(first), bits(planned))
+    wide = c.run(lambda: vb.launch_row_owned_wide_b(view, schedule, c.b_dev, c.c_dev, rhs, c.stream))
+    np.testing.assert_array_equal(bits(wide), bits(first))
+    schedule.long_count = 0
+    c.check_tolerance(c.run(lambda: vb.launch_row_owned(view, schedule, c.b_dev, c.c_dev, rhs, c.stream)), "whole")
+    c.close()
+
+
+def test_long_rows_from_a_graph_and_on_two_streams():
+    """The three kernels keep their state in the call's own C: a captured graph replays them, each replay between eager
+    calls on another stream with another B and C, and every result equals its first eager run."""
+    parity.note("long rows: graph and streams")
+    rhs = 16
+    c = parity.Case(skewed(700, 16, 150), rhs, 47)
+    plan = vb.Plan(c.matrix, rhs)
+    assert plan.launch_count() == 3
+    first = torch.from_numpy(c.run_plan(plan)).to(parity.DEVICE)
+    other_b = torch.from_numpy(o.make_random_input(c.host.scalar_cols * rhs, 48)).to(parity.DEVICE)
+    other_c = torch.empty_like(c.c_dev)
+    streams = [torch.cuda.Stream(device=parity.DEVICE) for _ in range(2)]
+    plan.execute(other_b, other_c, streams[1])
+    torch.cuda.synchronize()
+    other_first = other_c.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        plan.execute(c.b_dev, c.c_dev, streams[0])
+    for _ in range(5):
+        c.c_dev.fill_(float("nan"))
+        other_c.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            graph.replay()
+        plan.execute(other_b, other_c, streams[1])
+        torch.cuda.synchronize()
+        assert torch.equal(c.c_dev, first) and torch.equal(other_c, other_first)
+    plan.close()
+    c.close()
