@@ -407,7 +407,7 @@ void check_skewed(int32_t light, int32_t heavy, int32_t blocks, bool expected) {
   vbsr_host_view m = h.view();
   m.values_len = h.value_off.back();
   check_long_rows(m, vbsr_amd::build_schedule(m), expected);
-  std::printf("%s skewed: %d light, %d of %d blocks\n", failures == before ? "ok" : "FAILED", light, heavy, blocks);
+  std::printf("skewed: %d light, %d of %d blocks %s\n", light, heavy, blocks, failures == before ? "ok" : "FAILED");
 }
 
 // reorders: the matrix is random enough that a chained order must differ
