@@ -14,28 +14,30 @@
 // chain.  Tiles are transposed, D[n][r] = sum_k B[k, n] * A[r, k]: MFMA i of a
 // step at k0 takes k0 + 4 i .. k0 + 4 i + 3, lane 16 g + x supplying
 // B[k0 + 4 i + g, n0 + x] and A[r0 + x, k0 + 4 i + g], and result register v
-// of that lane is C[r0 + x, n0 + 4 g + v].  A step is 16 columns of a block;
-// the 8 columns that end a block whose width is 8 mod 16 take two MFMAs
-// instead of four, so no zero is ever added to a chain.
+// of that lane is C[r0 + x, n0 + 4 g + v].  A step is up to 32 columns of
+// a block, and takes two MFMAs for each 8 of them, so that no zero is ever
+// added to a chain.
 //
 // Mapping.  One workgroup of 4 waves per block row.  An output's chain cannot
 // be split, so the waves share the row's 16 x 16 output tiles instead: at
 // RHS 64 wave w takes RHS tile w of every row tile, at RHS 32 RHS tile w & 1
 // of every other row tile, at RHS 16 and 8 row tile w.  A step's A columns
-// (contiguous, 64 h bytes) and its B slice are loaded once per workgroup, 16
-// and RHS / 4 bytes per thread, kStages - 1 steps ahead in registers, and go
+// (contiguous, up to 8 KB) and its B slice (up to 128 bytes of each column at
+// once) are loaded once per workgroup, a step ahead in registers, and go
 // through two LDS buffers with one barrier per step.  Block metadata is read
 // 64 blocks at a time, one per lane.
 //
 // What bounds it.  At full size the L2-miss reads, as for the MFMA plan
-// kernel, whose time it comes within 7-22% of; for few, long rows one row's
-// chain of steps (0.36 us a step on an otherwise idle CU).  Measured at 4096
-// block rows of degree 8 (high sizes, random columns), against one fmaf per
-// output, k and lane with B broadcast from LDS, which the LDS read rate bound:
-// RHS 8 / 16 / 32 / 64 83.5 -> 42.8, 99.9 -> 47.6, 186 -> 65.1, 297 -> 106 us
-// per call.  Two stages: 300 rows of degree 16 +11%, the rest within 1%; four
-// stages: +1-3%.  Reading the next step's operands back from LDS during the
-// current step's MFMAs: -0.5% to +4%.
+// kernel, whose time it comes within 14-18% of; for few, long rows one row's
+// chain of steps.  Measured at 4096 block rows of degree 8 (high sizes, random
+// columns), against one fmaf per output, k and lane with B broadcast from LDS,
+// which the LDS read rate bound: RHS 8 / 16 / 32 / 64 83.5 -> 41.6, 99.9 ->
+// 46.5, 186 -> 63.6, 297 -> 104 us per call.  Steps of 16 columns instead of 32
+// (half the bytes a load, twice the barriers): +3% there, +5% with 32 x 32
+// blocks in a band, +12% at 300 rows of degree 16, but -4% at degree 1.  Three
+// stages instead of two: +1-3%, at degree 1 +9%, though -11% where one row of
+// 300 blocks is most of the launch.  Reading the next step's operands back from
+// LDS during the current step's MFMAs: -0.5% to +4%.
 #include <hip/hip_runtime.h>
 
 #include "../internal.hpp"
@@ -49,7 +51,8 @@ using rsrc_t = __amdgpu_buffer_rsrc_t;
 constexpr int kWave = 64;
 constexpr int kWaves = 4;
 constexpr int kThreads = kWave * kWaves;
-constexpr int kStages = 3;     // register stages of a step's loads
+constexpr int kStages = 2;     // register stages of a step's loads
+constexpr int kStepK = 32;     // most columns of a step
 constexpr int kMaxTiles = 4;   // h <= 64
 constexpr int kRawBufferFlags = 0x00020000;
 constexpr int kNonTemporal = 2;
@@ -58,8 +61,10 @@ template <int RHS>
 struct Shape {
   static constexpr int kRhsTiles = RHS < 16 ? 1 : RHS / 16;
   static constexpr int kWavesPerTileColumn = kWaves / kRhsTiles;  // waves that share an RHS tile's row tiles
-  static constexpr int kBVec = RHS < 16 ? 1 : RHS / 16;           // floats of B per thread and step
-  static constexpr int kBFloats = 16 * 16 * kRhsTiles;
+  // Floats of B per thread, load and step.
+  static constexpr int kBVec = RHS == 8 ? 1 : RHS == 16 ? 2 : 4;
+  static constexpr int kBLoads = RHS == 64 ? 2 : 1;
+  static constexpr int kBFloats = kStepK * 16 * kRhsTiles;
 };
 
 // Leading dimension of the A buffer, float (r, k) at k * ld + r: 16 mod 64 or
@@ -69,13 +74,13 @@ template <int T>
 constexpr int a_ld() {
   return T == 1 ? 16 : T == 4 ? 80 : 48;
 }
-constexpr int kAFloats = 16 * a_ld<kMaxTiles>();
+constexpr int kAFloats = kStepK * a_ld<kMaxTiles>();
 
-// Float (k, n) of the B buffer: column-major, the four 16-byte pieces of a
-// column permuted by an XOR of n's bits 1-2, which keeps the writes (16 k of
-// consecutive columns) and the reads (4 k of 16 columns) free of conflicts.
+// Float (k, n) of the B buffer: column-major, the eight 16-byte pieces of a
+// column permuted by an XOR of n's upper bits, which keeps the writes (a
+// column's k one after another) and the reads (4 k of 16 columns) apart.
 __device__ __forceinline__ int b_index(int k, int n) {
-  return n * 16 + ((((k >> 2) ^ (n >> 1) ^ (n >> 2)) & 3) << 2) + (k & 3);
+  return n * kStepK + ((((k >> 2) ^ (n >> 1)) & 7) << 2) + (k & 3);
 }
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -112,29 +117,36 @@ __device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const flo
   const int x = lane & 15;
   const int tid = wave * kWave + lane;
 
-  // A: this thread's 16 bytes of the step's column-major h x 16 tile.  f / h
-  // is (f * ceil(2^16 / h)) >> 16, exact for f < 1024 and h a multiple of 8.
-  const uint32_t h_recip = (65536u + uint32_t(h) - 1u) / uint32_t(h);
-  const int f = 4 * tid;
-  const int fk = int((uint32_t(f) * h_recip) >> 16);
-  const int a_write = fk * ld + (f - fk * h);
-  const bool a_owner = f < 16 * h;
+  // A: this thread's 16 bytes of load q of the step's column-major tile.  f / h
+  // is (f * ceil(2^20 / h)) >> 20, exact for f < 2048 and h up to 64.
+  constexpr int kALoads = (16 * T * kStepK + 4 * kThreads - 1) / (4 * kThreads);
+  const uint32_t h_recip = ((1u << 20) + uint32_t(h) - 1u) / uint32_t(h);
+  int a_write[kALoads];
+  bool a_owner[kALoads];
+#pragma unroll
+  for (int q = 0; q < kALoads; ++q) {
+    const int f = 4 * kThreads * q + 4 * tid;
+    const int fk = int((uint32_t(f) * h_recip) >> 20);
+    a_write[q] = fk * ld + (f - fk * h);
+    a_owner[q] = f < kStepK * h;
+  }
 
-  // B: this thread's floats k .. k + kBVec - 1 of column n of the step.  A
-  // half step has no k >= 8: those threads read their column's lower half
-  // again, which no MFMA of the half step takes.
-  constexpr int kPerColumn = 16 / S::kBVec;
+  // B: this thread's floats k .. k + kBVec - 1 of column n of the step (and, at
+  // RHS 64, of column n + 32).  Threads past the step's k read its first
+  // columns again, which costs no line, and which no MFMA takes.
+  constexpr int kPerColumn = kStepK / S::kBVec;
   const int b_n = tid / kPerColumn;
   const int b_k = (tid % kPerColumn) * S::kBVec;
-  const int b_col = RHS < 16 ? b_n & (RHS - 1) : b_n;
-  const float* b_lane = b + int64_t(b_col) * a.scalar_cols + b_k;
-  const int b_back = b_k >= 8 ? 8 : 0;
-  const int b_write = b_index(b_k, b_n);
+  const float* b_lane = b + int64_t(b_n) * a.scalar_cols;
+  int b_write[S::kBLoads];
+#pragma unroll
+  for (int q = 0; q < S::kBLoads; ++q) b_write[q] = b_index(b_k, b_n + 32 * q);
   float* a_bufs = lds;
   float* b_bufs = lds + 2 * kAFloats;
-  int b_read[4];
+  const int b_col = 16 * rhs_tile + (RHS < 16 ? x & (RHS - 1) : x);
+  int b_read[kStepK / 4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) b_read[i] = b_index(4 * i + group, 16 * rhs_tile + x);
+  for (int i = 0; i < kStepK / 4; ++i) b_read[i] = b_index(4 * i + group, b_col);
   const int a_read = group * ld + 16 * first_tile + x;
 
   f32x4 acc[kOwn];
@@ -158,21 +170,26 @@ __device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const flo
     int64_t at_a = lane_value(a_off, 0), at_b = lane_value(b_off, 0);
     int at_w = __builtin_amdgcn_readlane(w, 0);
     struct Stage {
-      f32x4 a;
-      bvec b;
-      int mfmas;  // 4, 2 for a half step, 0 past the segment
+      f32x4 a[kALoads];
+      bvec b[S::kBLoads];
+      int pieces;  // of eight columns; 0 past the segment
     };
     // Loads the next step.  Past the segment's end the A resource is empty
     // and B reads the last block's first columns again; neither is used.
     auto issue = [&](Stage& st) {
-      const bool live = at < blocks;
-      const bool half = at_w - k0 == 8;
-      st.mfmas = !live ? 0 : half ? 2 : 4;
+      const int width = min(at_w - k0, kStepK);
+      st.pieces = at < blocks ? width >> 3 : 0;
       const rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.values + at_a + int64_t(k0) * h),
-                                                            short(0), st.mfmas * 4 * h * 4, kRawBufferFlags);
-      st.a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * tid, 0, kNonTemporal));
-      st.b = *reinterpret_cast<const typename BVec<S::kBVec>::unaligned*>(b_lane + at_b + k0 - (half ? b_back : 0));
-      k0 += 16;
+                                                            short(0), st.pieces * 8 * h * 4, kRawBufferFlags);
+#pragma unroll
+      for (int q = 0; q < kALoads; ++q)
+        st.a[q] = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * tid + 16 * kThreads * q, 0, kNonTemporal));
+      const float* from = b_lane + at_b + k0 + (b_k < width ? b_k : 0);
+#pragma unroll
+      for (int q = 0; q < S::kBLoads; ++q)
+        st.b[q] = *reinterpret_cast<const typename BVec<S::kBVec>::unaligned*>(from + int64_t(32 * q) * a.scalar_cols);
+      k0 += kStepK;
       if (k0 >= at_w) {
         ++at;
         k0 = 0;
@@ -189,8 +206,11 @@ __device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const flo
       float* as = a_bufs + parity * kAFloats;
       float* bs = b_bufs + parity * S::kBFloats;
       parity ^= 1;
-      if (a_owner) *reinterpret_cast<f32x4*>(as + a_write) = st.a;
-      *reinterpret_cast<bvec*>(bs + b_write) = st.b;
+#pragma unroll
+      for (int q = 0; q < kALoads; ++q)
+        if (a_owner[q]) *reinterpret_cast<f32x4*>(as + a_write[q]) = st.a[q];
+#pragma unroll
+      for (int q = 0; q < S::kBLoads; ++q) *reinterpret_cast<bvec*>(bs + b_write[q]) = st.b[q];
       __syncthreads();
       auto mfma = [&](int i) {
         const float bv = bs[b_read[i]];
@@ -199,11 +219,12 @@ __device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const flo
           if (T % kStride == 0 || first_tile + j * kStride < T)
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv, as[a_read + 4 * i * ld + 16 * j * kStride], acc[j], 0, 0, 0);
       };
-      mfma(0);
-      mfma(1);
-      if (st.mfmas > 2) {
-        mfma(2);
-        mfma(3);
+#pragma unroll
+      for (int p = 0; p < kStepK / 8; ++p) {
+        if (p < st.pieces) {
+          mfma(2 * p);
+          mfma(2 * p + 1);
+        }
       }
     };
     Stage s[kStages];
@@ -214,9 +235,9 @@ __device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const flo
       for (int q = 0; q < kStages; ++q) {
         issue(s[(q + kStages - 1) % kStages]);
         __builtin_amdgcn_sched_barrier(0);
-        if (s[q].mfmas > 0) compute(s[q]);
+        if (s[q].pieces > 0) compute(s[q]);
       }
-      more = s[0].mfmas > 0;
+      more = s[0].pieces > 0;
     }
   }
 
