@@ -31,13 +31,16 @@
 // kernel, whose time it comes within 14-18% of; for few, long rows one row's
 // chain of steps.  Measured at 4096 block rows of degree 8 (high sizes, random
 // columns), against one fmaf per output, k and lane with B broadcast from LDS,
-// which the LDS read rate bound: RHS 8 / 16 / 32 / 64 83.5 -> 41.6, 99.9 ->
-// 46.5, 186 -> 63.6, 297 -> 104 us per call.  Steps of 16 columns instead of 32
-// (half the bytes a load, twice the barriers): +3% there, +5% with 32 x 32
-// blocks in a band, +12% at 300 rows of degree 16, but -4% at degree 1.  Three
-// stages instead of two: +1-3%, at degree 1 +9%, though -11% where one row of
-// 300 blocks is most of the launch.  Reading the next step's operands back from
-// LDS during the current step's MFMAs: -0.5% to +4%.
+// which the LDS read rate bound: RHS 8 / 16 / 32 / 64 83.6 -> 40.4, 99.8 ->
+// 46.3, 186 -> 63.6, 298 -> 102 us per call; degree 1: 13.1 -> 11.2, 15.2 ->
+// 12.7, 28.4 -> 19.0, 57.6 -> 29.2 us.  Steps of 16 columns instead of 32 (half
+// the bytes a load, twice the barriers): +3%, +12% at 300 rows of degree 16.
+// At degree 1 a workgroup lives for a step or two, and what counts is how many
+// of them a CU holds: a padded A buffer (7 of them, not 8) cost 5-10% there,
+// and loading ahead of a row's only step 4%.  Three stages instead of two:
+// +1-3%, at degree 1 +9%, though -11% where one row of 300 blocks is most of
+// the launch.  Reading the next step's operands back from LDS during the
+// current step's MFMAs: -0.5% to +4%.
 #include <hip/hip_runtime.h>
 
 #include "../internal.hpp"
@@ -67,14 +70,12 @@ struct Shape {
   static constexpr int kBFloats = kStepK * 16 * kRhsTiles;
 };
 
-// Leading dimension of the A buffer, float (r, k) at k * ld + r: 16 mod 64 or
-// 48 mod 64, so that the four lane groups, which read four consecutive k, hit
-// four disjoint quarters of the banks.
-template <int T>
-constexpr int a_ld() {
-  return T == 1 ? 16 : T == 4 ? 80 : 48;
-}
-constexpr int kAFloats = kStepK * a_ld<kMaxTiles>();
+// Float (r, k) of the A buffer: 64 to a k, the four 16-row tiles permuted by an
+// XOR of k's low bits, so that the four lane groups, which read four consecutive
+// k, cover all banks without padding (8 workgroups a CU at RHS 8 and 16).
+constexpr int kLd = 16 * kMaxTiles;
+constexpr int kAFloats = kStepK * kLd;
+__device__ __forceinline__ int a_index(int k, int r) { return k * kLd + (r ^ ((k & 3) << 4)); }
 
 // Float (k, n) of the B buffer: column-major, the eight 16-byte pieces of a
 // column permuted by an XOR of n's upper bits, which keeps the writes (a
@@ -107,7 +108,6 @@ __device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const flo
                                             float* lds, int wave, int lane) {
   using S = Shape<RHS>;
   using bvec = typename BVec<S::kBVec>::type;
-  constexpr int ld = a_ld<T>();
   // Row tiles of one wave: first, first + kStride, ...
   constexpr int kStride = S::kWavesPerTileColumn;
   constexpr int kOwn = (T + kStride - 1) / kStride;
@@ -127,7 +127,7 @@ __device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const flo
   for (int q = 0; q < kALoads; ++q) {
     const int f = 4 * kThreads * q + 4 * tid;
     const int fk = int((uint32_t(f) * h_recip) >> 20);
-    a_write[q] = fk * ld + (f - fk * h);
+    a_write[q] = a_index(fk, f - fk * h);
     a_owner[q] = f < kStepK * h;
   }
 
@@ -147,7 +147,9 @@ __device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const flo
   int b_read[kStepK / 4];
 #pragma unroll
   for (int i = 0; i < kStepK / 4; ++i) b_read[i] = b_index(4 * i + group, b_col);
-  const int a_read = group * ld + 16 * first_tile + x;
+  int a_read[kOwn];
+#pragma unroll
+  for (int j = 0; j < kOwn; ++j) a_read[j] = a_index(group, 16 * ((first_tile + j * kStride) & (kMaxTiles - 1)) + x);
 
   f32x4 acc[kOwn];
 #pragma unroll
@@ -217,7 +219,7 @@ __device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const flo
 #pragma unroll
         for (int j = 0; j < kOwn; ++j)
           if (T % kStride == 0 || first_tile + j * kStride < T)
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv, as[a_read + 4 * i * ld + 16 * j * kStride], acc[j], 0, 0, 0);
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv, as[a_read[j] + 4 * i * kLd], acc[j], 0, 0, 0);
       };
 #pragma unroll
       for (int p = 0; p < kStepK / 8; ++p) {
@@ -228,6 +230,11 @@ __device__ __forceinline__ void ordered_row(const vbsr_device_view& a, const flo
       }
     };
     Stage s[kStages];
+    if (blocks == 1 && at_w <= kStepK) {  // a single step: nothing to load ahead
+      issue(s[0]);
+      compute(s[0]);
+      continue;
+    }
 #pragma unroll
     for (int q = 0; q < kStages - 1; ++q) issue(s[q]);
     for (bool more = true; more;) {
