@@ -28,7 +28,7 @@
 // 64 blocks at a time, one per lane.
 //
 // What bounds it.  At full size the L2-miss reads, as for the MFMA plan
-// kernel, whose time it comes within 14-18% of; for few, long rows one row's
+// kernel, whose time it comes within 14-17% of; for few, long rows one row's
 // chain of steps.  Measured at 4096 block rows of degree 8 (high sizes, random
 // columns), against one fmaf per output, k and lane with B broadcast from LDS,
 // which the LDS read rate bound: RHS 8 / 16 / 32 / 64 83.6 -> 40.4, 99.8 ->
